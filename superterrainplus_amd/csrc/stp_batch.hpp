@@ -66,9 +66,6 @@ namespace SuperTerrainPlus {
 		// needs tile >= 2 halo. 0 = every drop works on the heightmap in HBM with global atomics.
 		unsigned int ErosionTile;
 		unsigned int ErosionThreads; // threads of one tile workgroup: 256, 512 or 1024
-		// Run the drops' lives in two halves, each with a halo of half the lifetime (so tile >= 2 halo
-		// holds for smaller tiles); 1024 threads.
-		bool ErosionHalves = false;
 	};
 
 	namespace STPBatch {
@@ -204,10 +201,6 @@ namespace SuperTerrainPlus {
 		// The smallest valid tile with 1024 threads: the most workgroups per colour batch, which
 		// shortens a small batch (a few chunks) at some cost in throughput.
 		STPBatchTuning latencyTuning() const;
-		// Lets every later bind() choose the shape with the shortest erosion of its chunks: half lives
-		// where the tiles of one colour batch are at most one per CU, latencyTuning() otherwise. Until
-		// the next setTuning().
-		void tuneForLatency();
 
 		unsigned long long pixels() const noexcept;
 		unsigned long long drops() const noexcept { return this->Drops; }
@@ -215,8 +208,8 @@ namespace SuperTerrainPlus {
 
 	private:
 		// tile tables: 0 biome, 1 vertical filter, 2 horizontal filter, 3 blend, 4 drops,
-		// 5..8 erosion tiles of colour 0..3, 9..12 those of the second half of the drops' lives
-		static constexpr int TableCount = 13;
+		// 5..8 erosion tiles of colour 0..3
+		static constexpr int TableCount = 9;
 		struct STPTileRange {
 			unsigned int Begin[TableCount], End[TableCount];
 		};
@@ -234,7 +227,6 @@ namespace SuperTerrainPlus {
 		std::vector<STPTileRange> Range;
 		std::array<unsigned int, TableCount> TileCount {};
 		STPBatchTuning Tuning {};
-		bool PerBinding = false; // tuneForLatency
 		unsigned int ErosionTiles = 0u, ErosionHalo = 0u, ErosionLds = 0u;
 		unsigned long long Pixels = 0ull, Drops = 0ull;
 
@@ -255,8 +247,6 @@ namespace SuperTerrainPlus {
 		// tiled erosion: per drop its rank in its spawn tile and the tile-sorted drop list; per
 		// tile its drop count and first slot
 		STPSmartDeviceMemory::STPDevice<unsigned int> DropRank, DropBin, TileDrops, TileFirst;
-		// drops between the halves of their lives, by slot (ErosionHalves)
-		STPSmartDeviceMemory::STPDevice<float4> HalfMotion;
 		STPSmartDeviceMemory::STPDevice<unsigned short> Fixed, BiomeMap;
 		STPSmartDeviceMemory::STPDevice<unsigned int> VBin;
 		// filter line segments: per slot (segment of a line) and biome, the run summary of the
@@ -303,14 +293,8 @@ namespace SuperTerrainPlus {
 		void releaseGraphs() noexcept;
 		void init(const STPEnvironment::STPRainDropSetting& rain);
 		void buildTileTables(hipStream_t stream);
-		// LDS bytes of the tiled erosion's window (0 if the tiled erosion is impossible).
-		unsigned int erosionLdsBytes(const STPBatchTuning& tuning) const;
-		// cells a drop's accesses can reach beyond its tile in its life, or in half of it
-		unsigned int erosionHalo(bool halves) const;
-		STPBatchTuning bindingTuning(const std::vector<STPBatch::Chunk>& chunks) const;
-		void applyTuning(const STPBatchTuning& tuning);
-		void reserveHalves();
-		unsigned long long halfDrops() const noexcept;
+		// Window side bound and LDS bytes of the tiled erosion for a tile side (0 if impossible).
+		unsigned int erosionLdsBytes(unsigned int tile) const;
 		STPStage::ErosionArgs erosionArgs() const;
 		// the filter passes with per-biome registers (at most 8 biomes and 8 bins per pixel)
 		bool itemPath() const noexcept;

@@ -462,10 +462,11 @@ struct STPHeightfieldGenerator::STPImpl {
 		cap.Chunks = 1u;
 		cap.MaxSide = side;
 		auto batch = std::make_unique<STPHeightfieldBatch>(noise, biome, this->RainSetting, setting, cap);
-		if (batch->latencyTuning().ErosionTile == 0u) {
+		const STPBatchTuning tuning = batch->latencyTuning();
+		if (tuning.ErosionTile == 0u) {
 			return nullptr;
 		}
-		batch->tuneForLatency();
+		batch->setTuning(tuning);
 		this->Gate = STPSmartDeviceMemory::makeDevice<unsigned int>(2u);
 		STP_CHECK_HIP(hipEventCreateWithFlags(&this->EroderDone, hipEventDisableTiming));
 		this->Eroder = std::move(batch);

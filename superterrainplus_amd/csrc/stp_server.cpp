@@ -81,14 +81,9 @@ STPHeightfieldServer::STPHeightfieldServer(const STPEnvironment::STPSimplexNoise
 	this->Engines.resize(setting.Engines);
 	for (Engine& e : this->Engines) {
 		e.Batch = std::make_unique<STPHeightfieldBatch>(noise, biome, rain, batch, cap);
-		// A serving batch holds a few chunks, whose drops are spread over the most workgroups. The
-		// drops kept between half lives (32 bytes each) fit in the memory that packed histograms leave
-		// unused; with unpacked ones they would cost budget, and the smallest whole-life tile stays.
-		if (e.Batch->packedHistogram()) {
-			e.Batch->tuneForLatency();
-		} else {
-			e.Batch->setTuning(e.Batch->latencyTuning());
-		}
+		// a serving batch holds a few chunks: the smallest erosion tile spreads them over the most
+		// workgroups
+		e.Batch->setTuning(e.Batch->latencyTuning());
 		// default priority, non-blocking with respect to the null stream
 		STP_CHECK_HIP(hipStreamCreateWithFlags(&e.Stream, hipStreamNonBlocking));
 		STP_CHECK_HIP(hipEventCreateWithFlags(&e.Done, hipEventDisableTiming));

@@ -528,40 +528,27 @@ namespace SuperTerrainPlus::STPStage {
 		return r;
 	}
 
-	// A drop in parallel mode between its steps, and what it has counted so far.
-	struct DropRun {
-		DropState State;
-		float Lost;
-		unsigned int Steps, ErodeSteps, DepositSteps, Killed;
-	};
-	template <class Surface>
-	__device__ inline DropRun spawnRun(const Surface& s, const ErosionArgs& a, const unsigned int drop) {
-		DropRun r {spawn(a, drop), 0.0f, 0u, 0u, 0u, 0u};
-		if (!s.spawnGuard(a, r.State)) {
-			r.State.volume = 0.0f;
-			r.Killed = 1u;
-		}
-		return r;
-	}
-	// one past the last step of a drop's life
-	__device__ inline unsigned int lifetimeEnd(const ErosionArgs& a) {
-		return a.Rain.MaxLifetime == 0u ? 0xFFFFFFFFu : a.Rain.MaxLifetime;
-	}
-
-	// Steps [begin, end) of a drop in parallel mode on `s`, or up to its death. `brush` holds (linear
-	// tap offset for s.stride(), weight bits). Taps > 0 is the compile-time brush size, Taps == 0 a loop
-	// over a.BrushSize taps; the surface's `erode` does a step's erode update.
+	// One drop in parallel mode on `s`. `brush` holds (linear tap offset for s.stride(), weight
+	// bits). Taps > 0 is the compile-time brush size, Taps == 0 a loop over a.BrushSize taps; the
+	// surface's `erode` does a step's erode update. The drop's final sediment and counters go to
+	// ledger[slot] and drop_info[slot].
 	template <class Surface, unsigned int Taps>
-	__device__ inline void stepDrop(const Surface& s, const ErosionArgs& a, const int2* const brush, DropRun& r,
-		const unsigned int begin, const unsigned int end) {
-		DropState& d = r.State;
+	__device__ inline void erodeDrop(const Surface& s, const ErosionArgs& a, const int2* const brush,
+		const unsigned int drop, const unsigned int slot, float* const ledger, uint2* const drop_info) {
+		DropState d = spawn(a, drop);
+		float lost = 0.0f;
+		unsigned int steps = 0u, erodeSteps = 0u, depositSteps = 0u, killed = 0u;
+		if (!s.spawnGuard(a, d)) {
+			d.volume = 0.0f;
+			killed = 1u;
+		}
 		// the kill test's bounds, with the surface's own footprint test folded in where it has one
 		const float4 bounds = s.moveBounds(a);
 		// the drop's cell, carried from the step that moved the drop there
 		DropCell c = dropCell(s, d.px, d.py);
 		const float inertia = a.Rain.Inertia, gradientScale = (1 - inertia) * Surface::Unit;
-		for (unsigned int life = begin; life < end && d.volume >= a.Rain.minWaterVolume; life++) {
-			r.Steps++;
+		for (unsigned int life = 0u; alive(a, d, life); life++) {
+			steps++;
 			// unscaled: (-g Unit)(1 - inertia) = (-g)((1 - inertia) Unit) exactly
 			const float3 hg = surfaceGradient(s, c);
 			// STPRainDrop.cu:86-105 (direction, move, kill test)
@@ -581,10 +568,10 @@ namespace SuperTerrainPlus::STPStage {
 			const bool inMap = ((d.dx != 0.0f) | (d.dy != 0.0f)) & (d.px >= bounds.x) & (d.px < bounds.y)
 				& (d.py >= bounds.z) & (d.py < bounds.w);
 			if (!(inMap & s.stepGuard(a, c.X, c.Y))) {
-				r.Lost = d.sediment;
+				lost = d.sediment;
 				d.volume = 0.0f;
 				d.sediment = 0.0f;
-				r.Killed = 1u;
+				killed = 1u;
 				break;
 			}
 			const DropCell next = dropCell(s, d.px, d.py);
@@ -601,58 +588,24 @@ namespace SuperTerrainPlus::STPStage {
 				s.add(mapIndex + 1u, amount * ox * (1.0f - oy));
 				s.add(mapIndex + W, amount * (1.0f - ox) * oy);
 				s.add(mapIndex + W + 1u, amount * ox * oy);
-				r.DepositSteps++;
+				depositSteps++;
 			} else {
 				const float amount = fminf((cap - d.sediment) * a.Rain.ErodeSpeed, -deltaHeight);
 				d.sediment += s.template erode<Taps>(mapIndex, amount, brush, a.BrushSize);
-				r.ErodeSteps++;
+				erodeSteps++;
 			}
 			advance<true>(a, d, deltaHeight);
 			c = next;
 		}
-	}
-
-	// The drop's final sediment and counters go to ledger[slot] and drop_info[slot].
-	__device__ inline void finishDrop(const DropRun& r, const unsigned int slot, float* const ledger,
-		uint2* const drop_info) {
 		if (ledger) {
-			ledger[slot] = r.Lost + r.State.sediment;
+			ledger[slot] = lost + d.sediment;
 		}
 		if (drop_info) {
-			drop_info[slot] = packDropInfo(r.Steps, r.ErodeSteps, r.DepositSteps, r.Killed);
+			drop_info[slot] = packDropInfo(steps, erodeSteps, depositSteps, killed);
 		}
 	}
 
-	// One drop's whole life in parallel mode on `s`.
-	template <class Surface, unsigned int Taps>
-	__device__ inline void erodeDrop(const Surface& s, const ErosionArgs& a, const int2* const brush,
-		const unsigned int drop, const unsigned int slot, float* const ledger, uint2* const drop_info) {
-		DropRun r = spawnRun(s, a, drop);
-		stepDrop<Surface, Taps>(s, a, brush, r, 0u, lifetimeEnd(a));
-		finishDrop(r, slot, ledger, drop_info);
-	}
-
-	// Steps of a drop with any brush; brush sizes with a specialised (straight-line) step: r = 2, 3, 4.
-	template <class Surface>
-	__device__ inline void stepDropAnyBrush(const Surface& s, const ErosionArgs& a, const int2* const brush, DropRun& r,
-		const unsigned int begin, const unsigned int end) {
-		switch (a.BrushSize) {
-		case 9u:
-			stepDrop<Surface, 9u>(s, a, brush, r, begin, end);
-			break;
-		case 25u:
-			stepDrop<Surface, 25u>(s, a, brush, r, begin, end);
-			break;
-		case 45u:
-			stepDrop<Surface, 45u>(s, a, brush, r, begin, end);
-			break;
-		default:
-			stepDrop<Surface, 0u>(s, a, brush, r, begin, end);
-			break;
-		}
-	}
-
-	// One drop's whole life with any brush.
+	// Brush sizes with a specialised (straight-line) drop: r = 2, 3, 4.
 	template <class Surface>
 	__device__ inline void erodeDropAnyBrush(const Surface& s, const ErosionArgs& a, const int2* const brush,
 		const unsigned int drop, const unsigned int slot, float* const ledger, uint2* const drop_info) {
