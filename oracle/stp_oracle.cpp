@@ -277,7 +277,7 @@ void erodeSerial(Real* const map, const uint32_t totalX, const uint32_t totalY, 
 		// Spawn guard (build-defined): a spawn whose 2x2 bilinear cell leaves the map dies
 		// before its first step (the reference would read out of bounds there).
 		if (!(static_cast<uint32_t>(dr.px) + 1u <= totalX - 1u && static_cast<uint32_t>(dr.py) + 1u <= totalY - 1u)) {
-			dr.volume = Real(0);
+			dr.volume = Real(-1); // below every valid minWaterVolume, which may be 0
 			st.killed++;
 		}
 

@@ -59,7 +59,7 @@ namespace {
 			float lost = 0.0f;
 			unsigned int steps = 0u, erodeSteps = 0u, depositSteps = 0u, killed = 0u;
 			if (!spawnInside(a, d)) {
-				d.volume = 0.0f;
+				d.volume = DeadVolume;
 				killed = 1u;
 			}
 			for (unsigned int life = 0u; alive(a, d, life); life++) {

@@ -123,6 +123,10 @@ namespace SuperTerrainPlus::STPStage {
 			&& static_cast<unsigned int>(d.py) + 1u <= a.Total.y - 1u;
 	}
 
+	// Water volume of a drop that dies before its first step: below every valid minWaterVolume, which may
+	// be 0.
+	constexpr float DeadVolume = -1.0f;
+
 	// Fast = the hardware square root (1 ulp) of the parallel modes, which are assessed
 	// statistically; the serialized kernel keeps the correctly rounded sqrtf.
 	template <bool Fast = false>
@@ -539,7 +543,7 @@ namespace SuperTerrainPlus::STPStage {
 		float lost = 0.0f;
 		unsigned int steps = 0u, erodeSteps = 0u, depositSteps = 0u, killed = 0u;
 		if (!s.spawnGuard(a, d)) {
-			d.volume = 0.0f;
+			d.volume = DeadVolume;
 			killed = 1u;
 		}
 		// the kill test's bounds, with the surface's own footprint test folded in where it has one

@@ -59,7 +59,8 @@ def setting(drops, radius, lifetime, **kw):
 
 SPARSE = [(512, 1, 16, 3, 16, {}), (512, 1, 16, 3, 30, {}), (333, 1, 8, 2, 31, {}), (400, 1, 8, 4, 40, {}), (256, 1, 6, 1, 24, {}),
           (300, 1, 6, 5, 25, {}), (200, 3, 4, 3, 30, {}), (512, 1, 12, 3, 40, {"minWaterVolume": 0.75}),
-          (512, 1, 12, 3, 40, {"minWaterVolume": 0.9}), (96, 1, 1, 3, 30, {}), (64, 3, 1, 3, 30, {})]
+          (512, 1, 12, 3, 40, {"minWaterVolume": 0.9}), (96, 1, 1, 3, 40, {"minWaterVolume": 0.0}),
+          (512, 1, 12, 1, 40, {"minWaterVolume": 0.0}), (96, 1, 1, 3, 30, {}), (64, 3, 1, 3, 30, {})]
 
 
 @pytest.mark.parametrize("side,nn,drops,radius,lifetime,kw", SPARSE)

@@ -203,6 +203,17 @@ def test_erosion_flat_plane_kills_every_drop(oracle):
     assert stats[3] == 500 and stats[0] == stats[3]
 
 
+def test_erosion_spawn_outside_dies_at_once(oracle):
+    """A spawn whose cell leaves the map (u = 1: the last column, the last row) takes no step, also where
+    a drop may run dry."""
+    for seed in (16390493, 17845651):
+        for water in (0.0, 0.01):
+            h = np.tile(np.linspace(0.2, 0.5, 80, dtype=np.float32), (80, 1))
+            before = h.copy()
+            ledger, stats = oracle.erode(h, (1, 1), (80, 80), rain(oracle, 1, minWaterVolume=water), 1, seed)
+            assert (h == before).all() and ledger[0] == 0.0 and stats.tolist() == [0, 0, 0, 1]
+
+
 def test_erosion_tilted_plane_first_step(oracle):
     a = 0.001
     x = np.arange(64, dtype=np.float64)
