@@ -207,6 +207,15 @@ int stp_hydraulic_erosion(float* d_height, const stp_nn_information* nn, const s
 	const int32_t* d_brush_index, const float* d_brush_weight, uint32_t brush_size, uint32_t stream_id, int mode,
 	float* d_ledger, uint32_t* d_drop_info, void* stream);
 
+/* The form in which the generator runs mode 1, with drops that cannot meet run at the same time: the same
+ * heights bit for bit, for more than one drop, a MaxLifetime of 1 to 256, a brush radius of up to 16 and
+ * a map side of up to 65535. A wave waits at most poll_limit rounds for the drops before its own (the
+ * generator: 2^22, some seconds); after that the drops are run one after another and *gave_up is 1, else
+ * 0. Waits for the stream. */
+int stp_hydraulic_erosion_ordered(float* d_height, const stp_nn_information* nn, const stp_raindrop_setting* setting,
+	const int32_t* d_brush_index, const float* d_brush_weight, uint32_t brush_size, uint32_t stream_id, uint32_t poll_limit,
+	int* gave_up, void* stream);
+
 /* STPNearestNeighbourTextureBuffer merge / unmerge (SuperTerrain+/SuperTerrain+/Private/World/Chunk/
  * STPNearestNeighbourTextureBuffer.cpp:69-113) as device gather / scatter. h_chunk_ptrs is a host
  * array of NN.x * NN.y device pointers in row-major neighbour order; element_size is 1, 2 or 4. */

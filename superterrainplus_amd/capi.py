@@ -223,6 +223,8 @@ _SIGNATURES = {
     "stp_format_heightmap": (_I, [_P, _P, _U32, _U32, _P]),
     "stp_hydraulic_erosion": (_I, [_P, C.POINTER(NNInformation), C.POINTER(RainDropSetting), _P,
                                    _P, _U32, _U32, _I, _P, _P, _P]),
+    "stp_hydraulic_erosion_ordered": (_I, [_P, C.POINTER(NNInformation), C.POINTER(RainDropSetting), _P,
+                                           _P, _U32, _U32, _U32, C.POINTER(_I), _P]),
     "stp_nn_merge": (_I, [_P, _P, _U32, C.POINTER(NNInformation), _P]),
     "stp_nn_unmerge": (_I, [_P, _P, _U32, C.POINTER(NNInformation), _P]),
     "stp_voronoi_biomemap": (_I, [_U64, _U32, _U32, C.c_int64, C.c_int64, _P, _U32, _U32, _U32,

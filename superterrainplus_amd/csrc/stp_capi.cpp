@@ -439,6 +439,23 @@ int stp_format_heightmap(const float* const d_height, uint16_t* const d_fixed, c
 	});
 }
 
+namespace {
+	// The given brush must be the one generated for this map width and radius: the kernels' in-bounds
+	// argument holds for its taps only.
+	void checkBrush(const STPNearestNeighbourInformation& n, const STPEnvironment::STPRainDropSetting& r,
+		const int32_t* const d_brush_index, const float* const d_brush_weight, const uint32_t brush_size, const hipStream_t stream) {
+		std::vector<int> idx;
+		std::vector<float> w;
+		STPErosionBrushGenerator::generate(n.TotalMapSize.x, r.ErosionBrushRadius, idx, w);
+		require(brush_size == idx.size(), "brush size does not match the brush of this radius and map width");
+		require(d_brush_index != nullptr && d_brush_weight != nullptr, "null brush");
+		std::vector<int> given(idx.size());
+		STP_CHECK_HIP(hipMemcpyAsync(given.data(), d_brush_index, idx.size() * sizeof(int), hipMemcpyDeviceToHost, stream));
+		STP_CHECK_HIP(hipStreamSynchronize(stream));
+		require(given == idx, "brush indices differ from the brush of this radius and map width");
+	}
+}
+
 int stp_hydraulic_erosion(float* const d_height, const stp_nn_information* const nn, const stp_raindrop_setting* const setting,
 	const int32_t* const d_brush_index, const float* const d_brush_weight, const uint32_t brush_size,
 	const uint32_t stream_id, const int mode, float* const d_ledger, uint32_t* const d_drop_info, void* const stream) {
@@ -447,22 +464,28 @@ int stp_hydraulic_erosion(float* const d_height, const stp_nn_information* const
 		r.validate();
 		require(mode == 0 || mode == 1, "erosion mode must be 0 (parallel) or 1 (serialized)");
 		const STPNearestNeighbourInformation n = toNN(nn);
-		// the brush must be the one generated for this map width and radius (its extent is what
-		// the in-bounds argument of the kernel relies on)
-		std::vector<int> idx;
-		std::vector<float> w;
-		STPErosionBrushGenerator::generate(n.TotalMapSize.x, r.ErosionBrushRadius, idx, w);
-		require(brush_size == idx.size(), "brush size does not match the brush of this radius and map width");
-		// the kernel's in-bounds argument holds for this brush's taps only: check the indices
-		require(d_brush_index != nullptr && d_brush_weight != nullptr, "null brush");
-		std::vector<int> given(idx.size());
-		STP_CHECK_HIP(hipMemcpyAsync(given.data(), d_brush_index, idx.size() * sizeof(int), hipMemcpyDeviceToHost,
-			toStream(stream)));
-		STP_CHECK_HIP(hipStreamSynchronize(toStream(stream)));
-		require(given == idx, "brush indices differ from the brush of this radius and map width");
+		checkBrush(n, r, d_brush_index, d_brush_weight, brush_size, toStream(stream));
 		STPHeightfieldKernel::hydraulicErosion(d_height, n, toParam(r), d_brush_index, d_brush_weight, brush_size,
 			stream_id, static_cast<STPHeightfieldKernel::STPErosionMode>(mode), d_ledger,
 			reinterpret_cast<uint2*>(d_drop_info), toStream(stream));
+	});
+}
+
+int stp_hydraulic_erosion_ordered(float* const d_height, const stp_nn_information* const nn,
+	const stp_raindrop_setting* const setting, const int32_t* const d_brush_index, const float* const d_brush_weight,
+	const uint32_t brush_size, const uint32_t stream_id, const uint32_t poll_limit, int* const gave_up, void* const stream) {
+	return guarded([&] {
+		require(gave_up != nullptr, "null pointer");
+		const STPEnvironment::STPRainDropSetting r = toRain(setting);
+		r.validate();
+		const STPNearestNeighbourInformation n = toNN(nn);
+		checkBrush(n, r, d_brush_index, d_brush_weight, brush_size, toStream(stream));
+		require(STPHeightfieldKernel::orderedErosionApplies(n, toParam(r)),
+			"the ordered erosion takes several drops of a bounded lifetime and a small brush");
+		const auto workspace = STPSmartDeviceMemory::makeDevice<char>(STPHeightfieldKernel::orderedErosionBytes(n, toParam(r)));
+		STPHeightfieldKernel::orderedErosion(d_height, n, toParam(r), d_brush_index, d_brush_weight, brush_size, stream_id,
+			workspace.get(), toStream(stream), poll_limit);
+		*gave_up = STPHeightfieldKernel::orderedErosionGaveUp(workspace.get(), toStream(stream)) ? 1 : 0;
 	});
 }
 

@@ -90,12 +90,16 @@ namespace SuperTerrainPlus {
 			STPErosionMode mode, float* ledger, uint2* drop_info, hipStream_t stream, const unsigned int* gate = nullptr);
 		// the serialized mode with independent drops run at the same time: the same heights bit for bit,
 		// for erosions with a lifetime bound; `workspace` (orderedErosionBytes) is free again once
-		// `stream` has passed the call
+		// `stream` has passed the call. A wave that has waited `poll_limit` rounds gives up, and the drops
+		// are run one after another.
+		constexpr unsigned int OrderedPollLimit = 1u << 22; // seconds
 		bool orderedErosionApplies(const STPNearestNeighbourInformation& nn, const STPRainDropParameter& rd) noexcept;
 		size_t orderedErosionBytes(const STPNearestNeighbourInformation& nn, const STPRainDropParameter& rd);
 		void orderedErosion(float* height, const STPNearestNeighbourInformation& nn, const STPRainDropParameter& rd,
 			const int* brush_index, const float* brush_weight, unsigned int brush_size, unsigned int stream_id, void* workspace,
-			hipStream_t stream);
+			hipStream_t stream, unsigned int poll_limit = OrderedPollLimit);
+		// whether the call that used `workspace` gave up (waits for `stream`)
+		bool orderedErosionGaveUp(const void* workspace, hipStream_t stream);
 		void formatHeightmap(const float* input, STPHeightFixed_t* output, unsigned long long count, hipStream_t stream);
 		// gate[0] = 1 if a height of map[0, count) lies outside [low, high] or is NaN, else 0; gate[1] = 0
 		void heightGate(const float* map, unsigned long long count, float low, float high, unsigned int* gate,

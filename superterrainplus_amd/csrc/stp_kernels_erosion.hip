@@ -138,7 +138,7 @@ namespace {
 	//
 	// Every wait ends: drops are taken in index order by waves that are already running, a drop waits
 	// for lower indices only, and the lowest unfinished one waits for nobody. A wave that still
-	// polls after PollLimit rounds (seconds) raises the stop word, on which every wave leaves; the
+	// polls after `poll_limit` rounds raises the stop word, on which every wave leaves; the
 	// serialized kernel then erodes the saved map.
 	//
 	// What bounds it: the chain of drops in each other's way, each link a poll, a window load, the
@@ -150,7 +150,6 @@ namespace {
 	constexpr unsigned int OrderedSteps = 4u;   // steps of one chunk
 	constexpr unsigned int OrderedList = 2u * OrderedWaves;
 	constexpr unsigned int OrderedLifetime = 256u, OrderedRadius = 16u;
-	constexpr unsigned int PollLimit = 1u << 22;
 	// taps of the radius-16 brush (dx^2 + dy^2 < 256)
 	constexpr unsigned int OrderedTaps = 800u;
 
@@ -218,7 +217,7 @@ namespace {
 	// Taps: the brush size (9, 25 or 45: its sums are straight-line code), or 0 for any
 	template <unsigned int Taps>
 	__global__ void __launch_bounds__(64) orderedErosionKERNEL(float* const map, const ErosionArgs a, const int* const brush_index,
-		const float* const brush_weight, DropWord* const word, OrderedHeader* const header) {
+		const float* const brush_weight, DropWord* const word, OrderedHeader* const header, const unsigned int poll_limit) {
 		extern __shared__ float window[]; // side x side, the same as fetched, the taps' offsets and weights
 		__shared__ unsigned int before[OrderedList];
 		const unsigned int lane = threadIdx.x, r = a.Rain.ErosionBrushRadius, reach = orderedReach(r);
@@ -303,7 +302,7 @@ namespace {
 					if (__builtin_amdgcn_ballot_w64(blocked) == 0ull) {
 						break;
 					}
-					if (agentLoad(&header->Stop) != 0u || poll >= PollLimit) {
+					if (agentLoad(&header->Stop) != 0u || poll >= poll_limit) {
 						agentStore(&header->Stop, 1u);
 						return;
 					}
@@ -580,9 +579,16 @@ size_t STPHeightfieldKernel::orderedErosionBytes(const STPNearestNeighbourInform
 	return orderedSavedAt(rd.RainDropCount) + static_cast<size_t>(nn.TotalMapSize.x) * nn.TotalMapSize.y * sizeof(float);
 }
 
+bool STPHeightfieldKernel::orderedErosionGaveUp(const void* const workspace, const hipStream_t stream) {
+	OrderedHeader header;
+	STP_CHECK_HIP(hipMemcpyAsync(&header, workspace, sizeof(header), hipMemcpyDeviceToHost, stream));
+	STP_CHECK_HIP(hipStreamSynchronize(stream));
+	return header.Stop != 0u;
+}
+
 void STPHeightfieldKernel::orderedErosion(float* const height, const STPNearestNeighbourInformation& nn,
 	const STPRainDropParameter& rd, const int* const brush_index, const float* const brush_weight, const unsigned int brush_size,
-	const unsigned int stream_id, void* const workspace, const hipStream_t stream) {
+	const unsigned int stream_id, void* const workspace, const hipStream_t stream, const unsigned int poll_limit) {
 	const ErosionArgs a = erosionArguments(height, nn, rd, brush_index, brush_weight, brush_size, stream_id);
 	if (!workspace || !orderedErosionApplies(nn, rd) || brush_size > OrderedTaps) {
 		STP_THROW(STPInvalidArgument, "the ordered erosion does not take this map, brush or lifetime");
@@ -598,7 +604,7 @@ void STPHeightfieldKernel::orderedErosion(float* const height, const STPNearestN
 		lds = 2u * (side * side + brush_size) * static_cast<unsigned int>(sizeof(float));
 	const auto run = [&](auto kernel) {
 		kernel<<<rd.RainDropCount < OrderedWaves ? rd.RainDropCount : OrderedWaves, 64, lds, stream>>>(height, a, brush_index,
-			brush_weight, word, header);
+			brush_weight, word, header, poll_limit);
 	};
 	switch (brush_size) {
 	case 9u: run(orderedErosionKERNEL<9u>); break;

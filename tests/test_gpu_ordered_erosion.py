@@ -73,3 +73,40 @@ def test_ordered_erosion_bit_exact(gpu, oracle, mx, my, nn, drops, radius, lifet
     want = oracle.nn_unmerge(merged, (nn, nn), (mx, my))
     assert all(c.tobytes() == w.tobytes() for c, w in zip(chunks, want))
     assert all((f == w).all() for f, w in zip(fixed, oracle.nn_unmerge(oracle.format_heightmap(merged), (nn, nn), (mx, my))))
+
+
+def ordered(merged, mx, my, nn, rain, poll_limit):
+    """The heights of the ordered passes alone and whether they gave up."""
+    d = capi.DeviceArray.from_host(merged)
+    idx, w = capi.brush(mx * nn, rain.ErosionBrushRadius)
+    d_idx, d_w = capi.DeviceArray.from_host(idx), capi.DeviceArray.from_host(w)
+    gave_up = C.c_int(-1)
+    capi.call("stp_hydraulic_erosion_ordered", d.vp, C.byref(capi.nn_info((mx, my), (nn, nn))), C.byref(rain), d_idx.vp, d_w.vp,
+              idx.size, 0, poll_limit, C.byref(gave_up), None)
+    return d.download(), gave_up.value
+
+
+WAYS = [(64, 64, 1, 1500, 3, 30, {}), (96, 96, 3, 2000, 3, 30, {}), (128, 128, 1, 600, 2, 6, {}), (150, 170, 1, 150, 16, 12, {}),
+        (150, 150, 1, 200, 3, 256, {})]
+
+
+@pytest.mark.parametrize("limit", [1 << 22, 0])
+@pytest.mark.parametrize("mx,my,nn,drops,radius,lifetime,kw", WAYS)
+def test_ordered_passes_and_their_way_out(gpu, oracle, mx, my, nn, drops, radius, lifetime, kw, limit):
+    """The ordered passes come to their end by themselves. With no patience at all the first wave in another
+    one's way gives up, and the serialized kernel erodes the saved map. The oracle's bits both times."""
+    log(f"ordered passes {mx}x{my} nn={nn} drops={drops} r={radius} lifetime={lifetime} limit={limit}")
+    y, x = np.mgrid[0:my * nn, 0:mx * nn].astype(np.float64)
+    before = (0.5 + 0.2 * np.sin(x / 11.0) * np.cos(y / 17.0)).astype(np.float32)
+    rain = rain_setting(drops, radius, lifetime, **kw)
+    want = before.copy()
+    oracle.erode(want, (nn, nn), (mx, my), oracle_rain(oracle, rain), drops, rain.Seed, stream_id=0)
+    got, gave_up = ordered(before, mx, my, nn, rain, limit)
+    assert gave_up == (1 if limit == 0 else 0)
+    assert got.tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("drops,radius,lifetime", [(1, 3, 30), (60, 17, 30), (60, 3, 257)])
+def test_ordered_passes_refuse(gpu, drops, radius, lifetime):
+    with pytest.raises(capi.STPError):
+        ordered(np.full((90, 90), 0.5, np.float32), 90, 90, 1, rain_setting(drops, radius, lifetime), 1 << 22)
