@@ -200,8 +200,13 @@ struct STPSingleHistogramFilter::STPFilterBuffer::STPImpl {
 	size_t HostBinCapacity = 0u;
 	STPSmartDeviceMemory::STPHost<unsigned int> HostOffset;
 	size_t HostOffsetCapacity = 0u;
-	STPSmartDeviceMemory::STPHost<unsigned int> Flag; // {overflow, bin total}
-	STPSmartDeviceMemory::STPHost<STPHeightfieldKernel::STPLaneFilterReport> Report;
+	// what the device reports of a call
+	struct STPReport {
+		STPHeightfieldKernel::STPLaneFilterReport Lanes;
+		unsigned int Overflow, Bins; // of the line-by-line passes
+	};
+	STPSmartDeviceMemory::STPHost<STPReport> Report;
+	bool Crowded = false; // the last map held more items than the lane-per-item passes take
 	STPSingleHistogram Result {nullptr, nullptr};
 	size_t BinCount = 0u, OffsetCount = 0u;
 	hipStream_t OwnStream = nullptr;
@@ -223,8 +228,7 @@ STPSingleHistogramFilter::STPFilterBuffer::STPFilterBuffer(const STPExecutionTyp
 	}
 	this->Impl->Type = type;
 	this->Impl->Capacity = bin_capacity;
-	this->Impl->Flag = STPSmartDeviceMemory::makeHost<unsigned int>(2u);
-	this->Impl->Report = STPSmartDeviceMemory::makeHost<STPHeightfieldKernel::STPLaneFilterReport>(1u);
+	this->Impl->Report = STPSmartDeviceMemory::makeHost<STPImpl::STPReport>(1u);
 }
 
 STPSingleHistogramFilter::STPFilterBuffer::STPFilterBuffer(STPFilterBuffer&&) noexcept = default;
@@ -268,6 +272,7 @@ STPSingleHistogram STPSingleHistogramFilter::filterDevice(const STPSample_t* con
 	const hipStream_t stream) {
 	const uint2 start = STPHeightfieldKernel::checkFilterDomain(nn, radius);
 	STPFilterBuffer::STPImpl& b = *filter_buffer.Impl;
+	STPFilterBuffer::STPImpl::STPReport& found = b.Report[0];
 	const size_t pixels = static_cast<size_t>(nn.MapSize.x) * nn.MapSize.y;
 	const auto workspace = [&b, stream](const size_t need) {
 		if (need > b.WorkspaceBytes) {
@@ -289,26 +294,36 @@ STPSingleHistogram STPSingleHistogramFilter::filterDevice(const STPSample_t* con
 		return b.Result;
 	};
 	// One lane per item first: a 512^2 map of 15 ids at random, radius 32, takes 20.4 ms line by line
-	// (one lane per line, its bins searched one after another) and 0.10 ms here; a map of more
-	// items than the workspace holds lanes for is found out on the device and goes line by line.
-	if (STPHeightfieldKernel::laneFilterApplies(nn.MapSize, radius)) {
-		char* const ws = workspace(STPHeightfieldKernel::laneFilterBytes(nn.MapSize, radius, b.Capacity));
-		const STPSingleHistogram histogram = STPHeightfieldKernel::laneFilter(samplemap, nn.TotalMapSize.x, start, nn.MapSize,
-			radius, b.Capacity, ws, b.Report.get(), stream);
+	// (one lane per line, its bins searched one after another) and 0.10 ms here. A map of more items than
+	// the workspace holds lanes for is found out on the device and goes line by line; the buffer's next map
+	// then goes line by line too and has its items counted beside that, until one would have fitted (64^2
+	// with 88 items: 487 us line by line alone, 510 to 522 with a try before it, 499 with the count).
+	const uint2 map = nn.MapSize;
+	const bool applies = STPHeightfieldKernel::laneFilterApplies(map, radius, b.Capacity);
+	if (applies && !b.Crowded) {
+		char* const ws = workspace(STPHeightfieldKernel::laneFilterBytes(map, radius, b.Capacity));
+		const STPSingleHistogram histogram = STPHeightfieldKernel::laneFilter(samplemap, nn.TotalMapSize.x, start, map,
+			radius, b.Capacity, ws, &found.Lanes, stream);
 		STP_CHECK_HIP(hipStreamSynchronize(stream));
-		const STPHeightfieldKernel::STPLaneFilterReport& report = b.Report[0];
-		if (STPHeightfieldKernel::laneFilterHolds(report, b.Capacity)) {
-			return finish(report.Overflow != 0u, report.Bins, histogram);
+		if (found.Lanes.Held != 0u) {
+			return finish(found.Lanes.Overflow != 0u, found.Lanes.Bins, histogram);
 		}
 	}
-	const STPFilterWorkspace carved = STPHeightfieldKernel::carveFilterWorkspace(
-		workspace(STPHeightfieldKernel::filterWorkspaceBytes(nn.MapSize, radius, b.Capacity)), nn.MapSize, radius, b.Capacity);
-	STPHeightfieldKernel::singleHistogramFilter(samplemap, nn.TotalMapSize.x, start, nn.MapSize, radius, b.Capacity, true,
-		carved, stream);
-	STP_CHECK_HIP(hipMemcpyAsync(b.Flag.get(), carved.Overflow, sizeof(unsigned int), hipMemcpyDeviceToHost, stream));
-	STP_CHECK_HIP(hipMemcpyAsync(b.Flag.get() + 1, carved.Offset + pixels, sizeof(unsigned int), hipMemcpyDeviceToHost, stream));
+	char* const ws = workspace(STPHeightfieldKernel::LaneItemBytes
+		+ STPHeightfieldKernel::filterWorkspaceBytes(map, radius, b.Capacity));
+	found.Lanes.Held = 0u;
+	if (applies && b.Crowded) {
+		STPHeightfieldKernel::laneFilterItems(samplemap, nn.TotalMapSize.x, start, map, radius, b.Capacity, ws, stream);
+		STPHeightfieldKernel::laneFilterReport(map, radius, b.Capacity, ws, &found.Lanes, stream);
+	}
+	const STPFilterWorkspace carved = STPHeightfieldKernel::carveFilterWorkspace(ws + STPHeightfieldKernel::LaneItemBytes, map,
+		radius, b.Capacity);
+	STPHeightfieldKernel::singleHistogramFilter(samplemap, nn.TotalMapSize.x, start, map, radius, b.Capacity, true, carved, stream);
+	STP_CHECK_HIP(hipMemcpyAsync(&found.Overflow, carved.Overflow, sizeof(unsigned int), hipMemcpyDeviceToHost, stream));
+	STP_CHECK_HIP(hipMemcpyAsync(&found.Bins, carved.Offset + pixels, sizeof(unsigned int), hipMemcpyDeviceToHost, stream));
 	STP_CHECK_HIP(hipStreamSynchronize(stream));
-	return finish(b.Flag[0] != 0u, b.Flag[1], STPSingleHistogram {carved.Bin, carved.Offset});
+	b.Crowded = applies && found.Lanes.Held == 0u;
+	return finish(found.Overflow != 0u, found.Bins, STPSingleHistogram {carved.Bin, carved.Offset});
 }
 
 STPSingleHistogram STPSingleHistogramFilter::operator()(const STPSample_t* const samplemap,

@@ -151,21 +151,28 @@ namespace SuperTerrainPlus {
 			hipStream_t stream);
 
 		// --- single histogram filter with one lane per item (stp_kernels_shf_lanes.hip): the jagged
-		// histogram of singleHistogramFilter for windows of at most LaneItems distinct items
+		// histogram of singleHistogramFilter for windows of at most LaneItems distinct items (fewer on
+		// maps whose workspace would be large). Its workspace starts with LaneItemBytes of numbered items.
 		constexpr unsigned int LaneItems = 64u, LaneFilterRadius = 510u;
-		// What a call found, written by the device into `report` (pinned host memory): distinct items of
-		// the window, whether a histogram outgrew the bin capacity, bins of all pixels.
+		constexpr size_t LaneItemBytes = 65536u + 65536u / 8u + 512u;
+		// What a call found, written by the device into `report` (pinned host memory): whether the
+		// workspace held the window's distinct items (if not, nothing else was written), whether a
+		// histogram outgrew the bin capacity, bins of all pixels.
 		struct STPLaneFilterReport {
-			unsigned int Items, Overflow, Bins;
+			unsigned int Held, Overflow, Bins;
 		};
 		// whether the passes take a map of this size and radius
-		bool laneFilterApplies(uint2 map_size, unsigned int radius) noexcept;
+		bool laneFilterApplies(uint2 map_size, unsigned int radius, unsigned int bin_capacity);
 		size_t laneFilterBytes(uint2 map_size, unsigned int radius, unsigned int bin_capacity);
-		// whether the workspace held the window's items; if not, nothing but the report was written
-		bool laneFilterHolds(const STPLaneFilterReport& report, unsigned int bin_capacity) noexcept;
-		// arguments as singleHistogramFilter; the jagged arrays live in `workspace` (laneFilterBytes)
+		// Arguments as singleHistogramFilter. laneFilterItems numbers the items of the window,
+		// laneFilter follows it with the passes; the jagged arrays live in `workspace` (laneFilterBytes).
+		void laneFilterItems(const STPSample_t* sample, unsigned int pitch, uint2 start, uint2 map_size, unsigned int radius,
+			unsigned int bin_capacity, void* workspace, hipStream_t stream);
 		STPAlgorithm::STPSingleHistogram laneFilter(const STPSample_t* sample, unsigned int pitch, uint2 start, uint2 map_size,
 			unsigned int radius, unsigned int bin_capacity, void* workspace, STPLaneFilterReport* report, hipStream_t stream);
+		// laneFilterItems' verdict on its own, into report->Held once `stream` has passed the call
+		void laneFilterReport(uint2 map_size, unsigned int radius, unsigned int bin_capacity, const void* workspace,
+			STPLaneFilterReport* report, hipStream_t stream);
 
 	} // namespace STPHeightfieldKernel
 } // namespace SuperTerrainPlus

@@ -25,6 +25,8 @@
 // marking 13 -> 5 us).
 #include "stp_internal.hpp"
 
+#include <algorithm>
+
 using namespace SuperTerrainPlus;
 using namespace SuperTerrainPlus::STPHeightfieldKernel;
 
@@ -604,7 +606,7 @@ namespace {
 		}
 		if (threadIdx.x == 0u) {
 			a.Offset[static_cast<size_t>(a.Width) * a.Height] = carry;
-			report->Items = items;
+			report->Held = items <= a.Lanes ? 1u : 0u;
 			report->Overflow = a.Header->Overflow;
 			report->Bins = carry;
 		}
@@ -685,10 +687,15 @@ namespace {
 		return s;
 	}
 
-	// Lanes the workspace holds per line: twice the bin capacity, since the items of a whole map are
-	// often more than those of one window, from 16 to 64.
-	unsigned int workspaceLanes(const unsigned int bin_capacity) {
-		return bin_capacity <= 8u ? 16u : (bin_capacity <= 16u ? 32u : LaneItems);
+	// Lanes the workspace holds per line: 64 while the cells take at most a gigabyte (8 M pixels), on
+	// larger maps twice the bin capacity (the items of a whole map are often more than those of one window),
+	// from 16 to 64. A map of more items is found out on the device and goes line by line after all: 32^2 with
+	// 24 items takes 51 us here, 145 line by line, and took 181 where the workspace held 16 lanes.
+	constexpr size_t LaneCellBytes = 1ull << 30u;
+	unsigned int workspaceLanes(const uint2 map, const unsigned int quads, const unsigned int bin_capacity) {
+		const size_t cells = static_cast<size_t>(map.y) * quads * 4u * sizeof(unsigned short);
+		return cells * LaneItems <= LaneCellBytes ? LaneItems
+			: (bin_capacity <= 8u ? 16u : (bin_capacity <= 16u ? 32u : LaneItems));
 	}
 
 	// Places in the workspace; fills every field but the sample map's.
@@ -706,7 +713,7 @@ namespace {
 		a.Quads = (a.Columns + 3u) / 4u;
 		a.Capacity = cap;
 		a.ColumnCapacity = cap < 2u * radius + 1u ? cap : 2u * radius + 1u;
-		a.Lanes = workspaceLanes(cap);
+		a.Lanes = workspaceLanes(map, a.Quads, cap);
 		a.SegRows = segmentLength(a.Columns, map.y, radius);
 		a.SegColumns = segmentLength(map.y, map.x, radius);
 		a.Segs = (map.x + a.SegColumns - 1u) / a.SegColumns;
@@ -716,6 +723,8 @@ namespace {
 		a.Header = reinterpret_cast<LaneHeader*>(take(sizeof(LaneHeader)));
 		a.Id = reinterpret_cast<unsigned char*>(take(65536u));
 		a.Item = reinterpret_cast<unsigned short*>(take(LaneItems * sizeof(unsigned short)));
+		static_assert(BitmapWords * sizeof(unsigned int) + 65536u + 512u == LaneItemBytes && sizeof(LaneHeader) <= 256u
+			&& LaneItems * sizeof(unsigned short) <= 256u, "the numbered items come first");
 		a.RowSummary = reinterpret_cast<Summary*>(take(static_cast<size_t>(rowSegs) * a.Columns * a.Lanes * sizeof(Summary)));
 		a.ColumnSummary = reinterpret_cast<Summary*>(take(static_cast<size_t>(a.Segs) * map.y * a.Lanes * sizeof(Summary)));
 		a.Cell = reinterpret_cast<unsigned short*>(take(static_cast<size_t>(map.y) * a.Quads * 4u * a.Lanes * sizeof(unsigned short)));
@@ -729,41 +738,71 @@ namespace {
 
 } // namespace
 
-bool STPHeightfieldKernel::laneFilterApplies(const uint2 map_size, const unsigned int radius) noexcept {
-	// positions (and window counts) of a line in 16 bits; grids of at most 65535 segments
-	return radius <= LaneFilterRadius && map_size.x + 2u * radius < NoPosition && map_size.y + 2u * radius < NoPosition;
-}
-
 size_t STPHeightfieldKernel::laneFilterBytes(const uint2 map_size, const unsigned int radius, const unsigned int bin_capacity) {
 	LaneArgs a {};
 	return carve(nullptr, map_size, radius, bin_capacity, a);
 }
 
-bool STPHeightfieldKernel::laneFilterHolds(const STPLaneFilterReport& report, const unsigned int bin_capacity) noexcept {
-	return report.Items <= workspaceLanes(bin_capacity);
+bool STPHeightfieldKernel::laneFilterApplies(const uint2 map_size, const unsigned int radius, const unsigned int bin_capacity) {
+	// Positions (and window counts) of a line in 16 bits; grids of at most 65535 segments. A workspace beyond
+	// 64 GiB is only taken where the line-by-line passes take as much (bin capacities of 1 to 3 take less).
+	return radius <= LaneFilterRadius && map_size.x + 2ull * radius < NoPosition && map_size.y + 2ull * radius < NoPosition
+		&& laneFilterBytes(map_size, radius, bin_capacity)
+			<= std::max<size_t>(64ull << 30u, filterWorkspaceBytes(map_size, radius, bin_capacity));
+}
+
+namespace {
+	LaneArgs laneArguments(const STPSample_t* const sample, const unsigned int pitch, const uint2 start, const uint2 map_size,
+		const unsigned int radius, const unsigned int bin_capacity, void* const workspace) {
+		STP_ASSERT_DOMAIN(radius > 0u && (radius & 1u) == 0u, "radius should be an positive even number");
+		STP_ASSERT_DOMAIN(radius <= start.x && radius <= start.y,
+			"radius is too large and will overflow nearest neighbour boundary");
+		if (bin_capacity == 0u || bin_capacity > MaxBinCapacity) {
+			STP_THROW(STPInvalidArgument, "histogram bin capacity must be in [1, 64]");
+		}
+		if (!sample || map_size.x == 0u || map_size.y == 0u || !workspace || !laneFilterApplies(map_size, radius, bin_capacity)) {
+			STP_THROW(STPInvalidArgument, "invalid sample map");
+		}
+		LaneArgs a {};
+		carve(static_cast<char*>(workspace), map_size, radius, bin_capacity, a);
+		a.Window = sample + static_cast<size_t>(start.y - radius) * pitch + (start.x - radius);
+		a.Pitch = pitch;
+		return a;
+	}
+
+	__global__ void laneReportKERNEL(const LaneArgs a, STPLaneFilterReport* const report) {
+		report->Held = a.Header->Items <= a.Lanes ? 1u : 0u;
+	}
+} // namespace
+
+void STPHeightfieldKernel::laneFilterItems(const STPSample_t* const sample, const unsigned int pitch, const uint2 start,
+	const uint2 map_size, const unsigned int radius, const unsigned int bin_capacity, void* const workspace,
+	const hipStream_t stream) {
+	const LaneArgs a = laneArguments(sample, pitch, start, map_size, radius, bin_capacity, workspace);
+	laneClearKERNEL<<<(BitmapWords + LaneBlock - 1u) / LaneBlock, LaneBlock, 0, stream>>>(a);
+	laneMarkKERNEL<<<dim3((a.Columns + LaneBlock - 1u) / LaneBlock, (a.Height + 2u * radius + MarkRows - 1u) / MarkRows), LaneBlock, 0,
+		stream>>>(a);
+	laneRankKERNEL<<<1, LaneBlock, 0, stream>>>(a);
+	STP_CHECK_HIP(hipGetLastError());
+}
+
+void STPHeightfieldKernel::laneFilterReport(const uint2 map_size, const unsigned int radius, const unsigned int bin_capacity,
+	const void* const workspace, STPLaneFilterReport* const report, const hipStream_t stream) {
+	LaneArgs a {};
+	carve(const_cast<char*>(static_cast<const char*>(workspace)), map_size, radius, bin_capacity, a);
+	laneReportKERNEL<<<1, 1, 0, stream>>>(a, report);
+	STP_CHECK_HIP(hipGetLastError());
 }
 
 STPAlgorithm::STPSingleHistogram STPHeightfieldKernel::laneFilter(const STPSample_t* const sample, const unsigned int pitch,
 	const uint2 start, const uint2 map_size, const unsigned int radius, const unsigned int bin_capacity, void* const workspace,
 	STPLaneFilterReport* const report, const hipStream_t stream) {
-	STP_ASSERT_DOMAIN(radius > 0u && (radius & 1u) == 0u, "radius should be an positive even number");
-	STP_ASSERT_DOMAIN(radius <= start.x && radius <= start.y,
-		"radius is too large and will overflow nearest neighbour boundary");
-	if (bin_capacity == 0u || bin_capacity > MaxBinCapacity) {
-		STP_THROW(STPInvalidArgument, "histogram bin capacity must be in [1, 64]");
+	if (!report) {
+		STP_THROW(STPInvalidArgument, "null report");
 	}
-	if (!sample || map_size.x == 0u || map_size.y == 0u || !workspace || !report || !laneFilterApplies(map_size, radius)) {
-		STP_THROW(STPInvalidArgument, "invalid sample map");
-	}
-	LaneArgs a {};
-	carve(static_cast<char*>(workspace), map_size, radius, bin_capacity, a);
-	a.Window = sample + static_cast<size_t>(start.y - radius) * pitch + (start.x - radius);
-	a.Pitch = pitch;
+	laneFilterItems(sample, pitch, start, map_size, radius, bin_capacity, workspace, stream);
+	const LaneArgs a = laneArguments(sample, pitch, start, map_size, radius, bin_capacity, workspace);
 	const unsigned int rowSegs = (a.Height + a.SegRows - 1u) / a.SegRows, columnBlocks = (a.Columns + ColumnBlock - 1u) / ColumnBlock;
-	laneClearKERNEL<<<(BitmapWords + LaneBlock - 1u) / LaneBlock, LaneBlock, 0, stream>>>(a);
-	laneMarkKERNEL<<<dim3((a.Columns + LaneBlock - 1u) / LaneBlock, (a.Height + 2u * radius + MarkRows - 1u) / MarkRows), LaneBlock, 0,
-		stream>>>(a);
-	laneRankKERNEL<<<1, LaneBlock, 0, stream>>>(a);
 	if (rowSegs > 1u) {
 		// segment 0 also holds the 2r rows before its first output
 		const unsigned int bytes = columnStride((a.SegRows + 2u * radius + 3u) / 4u * 4u) * ColumnBlock;

@@ -2,13 +2,15 @@
 weights and offsets at the edges of their groups (16, 32 and 64 items), segments (64 outputs) and
 column blocks (16 columns), windows longer and shorter than a segment, ids over the whole 16-bit
 range, more items than lanes (the line-by-line passes take over), and the capacity rule."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from superterrainplus_amd import capi
 
 from helpers import log
-from test_gpu_shf import FilterBuffer, host_filter
+from test_gpu_shf import BIN, FilterBuffer, device_filter, host_filter
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +57,44 @@ def test_lane_filter_capacity(gpu, oracle, cap, ok):
         with pytest.raises(capi.STPError) as e:
             host_filter(buf, sample, (3, 3), (w, h), r)
         assert e.value.code == 4
+
+
+def lane_path(out, w, h):
+    """Whether the lane-per-item passes made this histogram: their bins lie right after their offsets (256-byte
+    aligned), the line-by-line passes have a scan's sums between."""
+    return out.Bin - out.HistogramStartOffset == (4 * (w * h + 1) + 255) // 256 * 256
+
+
+def check_device(oracle, buf, m, w, h, r):
+    item, weight, off = oracle.shf_window(m, (w, h), (w, h), r)
+    d = capi.DeviceArray.from_host(m)
+    out, n = device_filter(buf, d, (3, 3), (w, h), r)
+    bins, offset = np.zeros(n, BIN), np.zeros(w * h + 1, np.uint32)
+    capi.call("stp_memcpy_async", capi.ptr(bins), C.c_void_p(out.Bin), bins.nbytes, None)
+    capi.call("stp_memcpy_async", capi.ptr(offset), C.c_void_p(out.HistogramStartOffset), offset.nbytes, None)
+    capi.synchronize()
+    assert (offset == off).all() and (bins["item"] == item).all() and bins["weight"].tobytes() == weight.tobytes()
+    return lane_path(out, w, h)
+
+
+@pytest.mark.parametrize("ids,cap,lanes", [(5, 8, True), (40, 8, True), (64, 12, True), (65, 12, False)])
+def test_lane_filter_path(gpu, oracle, ids, cap, lanes):
+    """Which passes take a map depends on its items, not on the bin capacity."""
+    log(f"lane filter path ids={ids} cap={cap}")
+    w, h, r = 48, 40, 2
+    m = np.zeros((3 * h, 3 * w), np.uint16)
+    # every id once in the window of samples, far enough apart that a pixel sees few
+    for k in range(ids):
+        m[h + 4 * (k // 11), w + 4 * (k % 11)] = k * 997 % 65536
+    assert check_device(oracle, FilterBuffer(cap), m, w, h, r) == lanes
+
+
+def test_lane_filter_after_a_crowded_map(gpu, oracle):
+    """A buffer whose last map held too many items goes line by line until a map would have fitted."""
+    w, h, r = 70, 50, 4
+    crowded, plain = sample_map(3, w, h, 400, 4, True), sample_map(4, w, h, 6, 4, True)
+    buf, way = FilterBuffer(40), []
+    for k, m in enumerate((plain, crowded, crowded, plain, plain, crowded, plain)):
+        log(f"lane filter after a crowded map {k}")
+        way.append(check_device(oracle, buf, m, w, h, r))
+    assert way == [True, False, False, False, True, False, False]
