@@ -154,7 +154,8 @@ void STPHeightfieldKernel::simplexHeightmap(const STPPermutation& perm, const No
 	// A small map is bound by one thread's chain of octaves, a large one by VALU issue and the staging of
 	// the tables: one or two pixels a thread take, with the format's launch, 8.6 or 9.4 us on 64^2, 9.0
 	// or 10.2 on 512^2, 13.3 or 14.3 on 724^2, 20.1 both on 1024^2, 220 or 208 us on 4096^2.
-	if (static_cast<unsigned long long>(width) * rows <= 1ull << 19u) {
+	// A grid holds 65536 tiles along y: a map of one or two columns can have more rows than one pixel a thread takes.
+	if (static_cast<unsigned long long>(width) * rows <= 1ull << 19u && rows <= TileY * 65536u) {
 		launch(simplexHeightmapKERNEL<1u>, 1u);
 	} else {
 		launch(simplexHeightmapKERNEL<PixelPerThread>, PixelPerThread);

@@ -1,5 +1,5 @@
 """The fractal heightmap with one and with two pixels a thread: the oracle's bits for maps below, at and past
-the size where the launch changes, with ragged edges."""
+the size where the launch changes, with ragged edges, and with the most rows of a grid of one pixel a thread."""
 import ctypes as C
 
 import numpy as np
@@ -12,7 +12,7 @@ from helpers import log
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("width,rows", [(1, 1), (65, 7), (63, 129), (1024, 512), (1024, 513), (727, 723)])
+@pytest.mark.parametrize("width,rows", [(1, 1), (65, 7), (63, 129), (1024, 512), (1024, 513), (727, 723), (1, 262144), (1, 300001)])
 def test_heightmap_bit_exact(gpu, oracle, width, rows):
     log(f"heightmap {width}x{rows}")
     table = capi.PermutationTable(42, W.DISTRIBUTION, W.GRADIENT_OFFSET, W.ENGINE_MT19937)
