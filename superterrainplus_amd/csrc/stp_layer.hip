@@ -766,9 +766,14 @@ void STPLayerBiomeFactory::plan(STPLayerPlan& plan, const std::vector<STPLayerMa
 			}
 		}
 	}
-	// any coordinate outside int is outside what the reference's int arithmetic can address
-	for (const Box& b : box) {
-		if (!b.empty() && (b.X0 < INT32_MIN || b.Z0 < INT32_MIN || b.X1 > INT32_MAX || b.Z1 > INT32_MAX)) {
+	// Any coordinate outside int is outside what the reference's int arithmetic can address; a Voronoi node
+	// also takes 2 from its coordinates, a scale node adds 1.
+	for (size_t i = 0u; i < n * count; i++) {
+		const Box& b = box[i];
+		const auto kind = static_cast<STPLayerKind>(m.Node[i / count].Kind);
+		const long long low = INT32_MIN + (kind == STPLayerKind::Voronoi ? 2ll : 0ll),
+			high = INT32_MAX - (kind == STPLayerKind::Scale ? 1ll : 0ll);
+		if (!b.empty() && (b.X0 < low || b.Z0 < low || b.X1 > high || b.Z1 > high)) {
 			STP_THROW(STPInvalidArgument, "biome map coordinates out of the int range");
 		}
 	}

@@ -37,3 +37,32 @@ def test_layer_maps_bit_exact(gpu, oracle, width, height, origins):
         capi.lib().stp_layer_factory_destroy(factory)
     chain = [oracle.layer_node(n.Kind, n.Salt, [p for p in n.Parent if p >= 0], n.Param, n.CacheSize) for n in nodes]
     assert (got == oracle.layer_biomemap(chain, 77, registry_tuple(registry), origins, width, height)).all()
+
+
+LOW, HIGH = -2 ** 31, 2 ** 31 - 1
+
+
+@pytest.mark.parametrize("origin,ok", [((LOW, 0), False), ((0, LOW + 1), False), ((LOW + 2, LOW + 2), True), ((HIGH - 4, HIGH - 3), True),
+                                       ((HIGH - 3, 0), False)])
+def test_layer_coordinate_ends(gpu, oracle, origin, ok):
+    """Where a Voronoi root's own arithmetic would leave int (x - 2), and where its last column does, the
+    map is refused on the host."""
+    log(f"layer coordinates {origin}")
+    # a continent node (0), a Voronoi node (4) on it
+    nodes = [capi.LayerNode(0, 0, (C.c_int32 * 2)(-1, -1), 5, 32), capi.LayerNode(4, 0, (C.c_int32 * 2)(0, -1), 7, 32)]
+    registry, factory = capi.demo_biome_registry(), C.c_void_p()
+    capi.call("stp_layer_factory_create", (capi.LayerNode * 2)(*nodes), 2, 77, C.byref(registry), 5, 4, C.byref(factory))
+    try:
+        out = capi.DeviceArray((4, 5), np.uint16)
+        go = lambda: capi.call("stp_layer_factory_generate_device", factory, out.vp, (C.c_int32 * 2)(*origin), 1, None)  # noqa: E731
+        if not ok:
+            with pytest.raises(capi.STPError):
+                go()
+            return
+        go()
+        capi.synchronize()
+        got = out.download()
+    finally:
+        capi.lib().stp_layer_factory_destroy(factory)
+    chain = [oracle.layer_node(n.Kind, n.Salt, [p for p in n.Parent if p >= 0], n.Param, n.CacheSize) for n in nodes]
+    assert (got[None] == oracle.layer_biomemap(chain, 77, registry_tuple(registry), [origin], 5, 4)).all()
